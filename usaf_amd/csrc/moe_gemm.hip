@@ -38,7 +38,7 @@
 // The grid is persistent: tiles (expert m-tile x n-tile) come from a
 // device-side list, walked per die so one expert's n-tiles share an L2; no
 // host sync is needed.
-#include "common.h"
+#include "moe_gemm.h"
 
 #include <type_traits>
 
@@ -47,7 +47,7 @@ namespace {
 
 // Tile: up to BM slots of one expert (10 MFMA row blocks of 32; empty blocks
 // are skipped) x BN output columns x BK contraction per LDS stage.
-constexpr int BM = 320, BN = 128, BK = 64;
+constexpr int BM = 320, BN = 128;
 constexpr int WM_SUB = BM / 32 / 2;    // 32-row blocks per M-wave (2 M-waves x 2 N-waves)
 constexpr int kThreads = 512;                // 4 multiply waves + 4 producer waves
 constexpr int A_CHUNKS = BM * BK / 8 / 256;  // 16-byte A chunks per producer thread per k-tile
@@ -59,54 +59,7 @@ constexpr size_t kSmemBytes = (size_t)2 * (BM + BN) * LDSW * 2 + (2 * (MAX_E + 1
 
 enum { BMODE_NK = 0, BMODE_KN = 1 };
 enum { BQ_Q4 = 0, BQ_DENSE16 = 1 };
-enum { EPI_STORE = 0, EPI_SWIGLU_FWD = 1, EPI_SWIGLU_BWD = 2 };
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
-
-struct GemmArgs {
-  const uint16_t* A;       // activations, 16-bit, row stride lda
-  int64_t lda;
-  const int32_t* a_rows;   // A row of slot m (nullptr: row m)
-  const uint8_t* wq;       // packed codes of the whole [E, w_rows, w_cols] weight
-  const uint32_t* wsz;     // per 128-element group: fp16 scale bits | fp16 zero bits << 16
-  const uint16_t* w16;     // dense 16-bit weight [E, w_rows, w_cols] (BQ == BQ_DENSE16)
-  const int32_t* w_slot;   // dense weights in an arena: expert e's [w_rows, w_cols] block is
-  int64_t n_slots;         //   block w_slot[e] (clamped to [0, n_slots)) of w16; nullptr: block e
-  int64_t w_rows, w_cols;  // per-expert weight matrix
-  int64_t N, K;            // output columns, contraction length
-  int64_t inter;           // I (SwiGLU epilogues)
-  const int32_t* offsets;  // [E+1]
-  int E;
-  uint16_t* out;  int64_t ldo;   // STORE: C; SWIGLU_FWD: act; SWIGLU_BWD: dgu
-  uint16_t* out2; int64_t ldo2;  // SWIGLU_FWD: gu
-  const uint16_t* aux; int64_t ld_aux;  // SWIGLU_BWD: saved gu
-  uint16_t* out_t;                // SWIGLU_FWD (4-bit DMA kernel): act also in the blocked slot-major
-  const int32_t* blk_table;       //   layout of blk_table (usaf_hip_blocked_layout), or nullptr
-  const uint32_t* ovl;            // 4-bit DMA kernel: overlay entries (usaf_hip_overlay_* layout), or nullptr
-  int64_t ovl_words;              //   and their count (checked against what the GEMM reads)
-  int w_frag;                     // dense weights (DW): 1 = each expert block in the GEMM's fragment order
-  int64_t w_blk_elems;            //   (usaf_hip_dequant_q4_slices_frag) of w_blk_elems elements; 0: w_rows * w_cols
-};
-
-// Workgroup barrier ordering LDS accesses only.  __syncthreads() also orders
-// global memory, which makes every wave drain its outstanding global loads
-// (s_waitcnt vmcnt(0)) at each barrier and exposes the full memory latency of
-// the prefetched k-steps; no thread here communicates through global memory.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// Block of the dense weight operand that holds expert e: e itself, or its
-// arena slot (clamped, so a stale table can give wrong weights but never an
-// access outside the arena).
-__device__ __forceinline__ int64_t weight_block(const GemmArgs& g, int e) {
-  if (g.w_slot == nullptr) return e;
-  const int64_t s = g.w_slot[e];
-  return s < 0 ? 0 : (s >= g.n_slots ? g.n_slots - 1 : s);
-}
 
 // ---- 4-bit -> 16-bit conversion (bit-identical to dequantize_4bit) ----------
 
@@ -127,12 +80,6 @@ __device__ __forceinline__ void dq_word(uint32_t w, f16x2 s2, f16x2 z2, uint32_t
   out[1] = (u2 & 0xFFFFu) | (u3 << 16);
   out[2] = (u0 >> 16) | (u1 & 0xFFFF0000u);
   out[3] = (u2 >> 16) | (u3 & 0xFFFF0000u);
-}
-
-__device__ __forceinline__ uint32_t h2_to_bf2(uint32_t h2) {
-  const f16x2 h = __builtin_bit_cast(f16x2, h2);
-  const f32x2 f = {(float)h.x, (float)h.y};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
 }
 
 // 32 codes (16 bytes, one group) -> 32 16-bit operands in natural order.
@@ -165,22 +112,6 @@ __device__ __forceinline__ float bits_to_f32(uint16_t b) {
 }
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
-
-// silu(x) = x / (1 + e^-x) with the hardware exp2 and reciprocal (about 1 ulp
-// of fp32 each, far below the 16-bit rounding that follows)
-__device__ __forceinline__ float silu_fast(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
-}
-
-template <int DT>
-__device__ __forceinline__ f32x16 mfma32(const u32x4 a, const u32x4 b, f32x16 c) {
-  if constexpr (DT == USAF_BF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c,
-                                                  0, 0, 0);
-}
 
 // Weight row r of expert e (NK, SWIGLU_FWD): tile row b of n-tile nt pairs gate
 // and up rows so that each wave holds 32 gate and the matching 32 up columns.
@@ -774,48 +705,6 @@ constexpr int NK_EPI_ELEMS = NK_EPI_ARR * 32 * NK_EPW;
 constexpr size_t kNkSmemBytes =
     (size_t)2 * NK_BM * LDSW * 2 + (size_t)4 * NK_EPI_ELEMS * 2 + (size_t)(2 * (MAX_E + 1) + NK_THREADS) * 4;
 
-// 8 codes of one 32-bit word (code 2i in the low nibble of byte i) -> 8 16-bit
-// weights in natural order, bit-identical to dequantize_4bit:
-// fp16(fp16(q * s) + z), then RNE bf16 for bf16 operands.
-template <int DT>
-__device__ __forceinline__ u32x4 dq8(uint32_t w, f16x2 s2, f16x2 z2) {
-#pragma clang fp contract(off)
-  const f16x2 mul = {(f16)1.0f, (f16)0.0625f};
-  const f16x2 sub = {(f16)-1024.0f, (f16)-64.0f};
-  uint32_t o[4];
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    // byte p in both halves: the low half keeps code 2p (bits 0-3), the high half
-    // code 2p+1 (bits 20-23), as fp16 1024 + q and 1024 + 16 q
-    const uint32_t t = __builtin_amdgcn_perm(w, w, 0x0C000C00u | ((uint32_t)p << 16) | (uint32_t)p);
-    const uint32_t bits = (t & 0x00F0000Fu) | 0x64006400u;
-    const f16x2 q = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, bits), mul, sub);  // exact codes
-    const f16x2 m = q * s2;
-    const f16x2 v = m + z2;
-    o[p] = __builtin_bit_cast(uint32_t, v);
-    if constexpr (DT == USAF_BF16) o[p] = h2_to_bf2(o[p]);
-  }
-  return u32x4{o[0], o[1], o[2], o[3]};
-}
-
-// Codes 2p, 2p+1 of a 32-bit code word (byte p) -> their two 16-bit weights
-// (dq8 for one pair).  v_perm places byte p under the fp16 exponent byte 0x64 in
-// both halves; the mask keeps code 2p in the low half (1024 + q) and code 2p+1
-// in the high half (1024 + 16 q).
-template <int DT>
-__device__ __forceinline__ uint32_t dq_pair(uint32_t w, int p, f16x2 s2, f16x2 z2) {
-#pragma clang fp contract(off)
-  const f16x2 mul = {(f16)1.0f, (f16)0.0625f};
-  const f16x2 sub = {(f16)-1024.0f, (f16)-64.0f};
-  const uint32_t t = __builtin_amdgcn_perm(0x64646464u, w, 0x04000400u | ((uint32_t)p << 16) | (uint32_t)p) & 0xFFF0FF0Fu;
-  const f16x2 q = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, t), mul, sub);  // exact codes
-  const f16x2 m = q * s2;
-  const f16x2 v = m + z2;
-  uint32_t o = __builtin_bit_cast(uint32_t, v);
-  if constexpr (DT == USAF_BF16) o = h2_to_bf2(o);
-  return o;
-}
-
 // One tile of the NK kernel with NRB (>= the tile's occupied row blocks) row
 // blocks computed.  Row blocks past the expert's slots multiply rows of the
 // staged tile that are never stored.
@@ -1173,11 +1062,9 @@ __global__ __launch_bounds__(NK_THREADS) void moe_gemm_nk_kernel(const GemmArgs 
 // tile's last steps and epilogue.
 // =====================================================================================
 constexpr int Q_BM = 256, Q_BN = 256, Q_THREADS = 512, Q_WAVES = Q_THREADS / 64;
-constexpr int Q_MAX_E = 255;
 constexpr int Q_A_BYTES = Q_BM * BK * 2;                 // activation rows of one k-step
 constexpr int Q_C_BYTES = Q_BN * BK / 2;                 // codes of one k-step
 constexpr int Q_Z_BYTES = Q_BN * 4;                      // scale|zero words of one k-step
-constexpr int Q_OVL_WORDS = 64;                          // overlay entries per wave and k-step
 constexpr int Q_O_BYTES = Q_WAVES * Q_OVL_WORDS * 4;     // overlay entries of one k-step
 constexpr int Q_STAGE = Q_A_BYTES + Q_C_BYTES + Q_Z_BYTES + Q_O_BYTES;
 constexpr int Q_A_LOADS = Q_A_BYTES / (16 * Q_THREADS);  // 4 x 16 B per thread
@@ -2119,13 +2006,15 @@ int check_ovl(const GemmArgs& g, int epi, const char* what) {
 
 // grad-input GEMMs on transposed 4-bit weights (always the LDS-DMA kernel)
 template <int EPI>
-int launch_q4t(const GemmArgs& g, int dt, int64_t max_tiles, int64_t a_rows_total, hipStream_t st, const char* what) {
+int launch_q4t(const GemmArgs& g, int dt, int64_t max_tiles, int64_t S, int64_t a_rows_total, hipStream_t st,
+               const char* what) {
   if (g.E > Q_MAX_E) return set_error(USAF_ERR_UNSUPPORTED, "%s: needs E <= %d", what, Q_MAX_E);
   if (((uintptr_t)g.A & 15) || g.lda % 8 != 0)
     return set_error(USAF_ERR_INVALID, "%s: activations must be 16-byte aligned rows", what);
   if (a_rows_total * g.lda * 2 >= ((int64_t)1 << 32) || (int64_t)g.E * g.w_rows * g.w_cols / 2 >= ((int64_t)1 << 32))
     return set_error(USAF_ERR_UNSUPPORTED, "%s: operands beyond 4 GiB", what);
   if (int rc = check_ovl(g, EPI, what)) return rc;
+  if (few_slots(g, EPI, true, S)) return launch_few(g, EPI, true, dt, S, st, what);
   int64_t blocks = (int64_t)device_cu_count();
   if (blocks > max_tiles) blocks = max_tiles;
   if (blocks < 1) blocks = 1;
@@ -2153,7 +2042,7 @@ bool dw_dma_ok(const GemmArgs& g, int64_t a_rows_total) {
 }
 
 template <int EPI>
-int launch_gemm_nk(const GemmArgs& g, int dt, int64_t max_tiles, int64_t a_rows_total, hipStream_t st,
+int launch_gemm_nk(const GemmArgs& g, int dt, int64_t max_tiles, int64_t S, int64_t a_rows_total, hipStream_t st,
                    const char* what) {
   if (a_rows_total * g.lda >= ((int64_t)1 << 31))
     return set_error(USAF_ERR_UNSUPPORTED, "%s: activation operand of %lld x %lld elements exceeds 2^31", what,
@@ -2168,6 +2057,7 @@ int launch_gemm_nk(const GemmArgs& g, int dt, int64_t max_tiles, int64_t a_rows_
                      "%s: an overlay needs the 4-bit LDS-DMA kernel (4-bit weights, 16-byte aligned activation rows, "
                      "K %% 128 == 0, E <= %d, operands below 4 GiB)", what, Q_MAX_E);
   if (int rc = check_ovl(g, EPI, what)) return rc;
+  if (dma && few_slots(g, EPI, false, S)) return launch_few(g, EPI, false, dt, S, st, what);
   const bool dw = dense && dw_dma_ok(g, a_rows_total);
   int rc;
   if (dt == USAF_BF16)
@@ -2297,7 +2187,7 @@ extern "C" int usaf_hip_moe_gate_up_fwd(const void* x, int64_t T_rows, int64_t H
     g.blk_table = blk_table;
   }
   const int64_t max_tiles = (S / NK_BM + E) * ((I + 127) / 128);
-  if (int rc = launch_gemm_nk<EPI_SWIGLU_FWD>(g, dtype, max_tiles, T_rows, as_stream(stream), "moe_gate_up_fwd")) return rc;
+  if (int rc = launch_gemm_nk<EPI_SWIGLU_FWD>(g, dtype, max_tiles, S, T_rows, as_stream(stream), "moe_gate_up_fwd")) return rc;
   if (act_blk && !fused_t)
     return usaf_hip_gather_transpose_blocked(act, I, nullptr, offsets, blk_table, S, E, I, act_blk, stream);
   return USAF_OK;
@@ -2322,7 +2212,7 @@ extern "C" int usaf_hip_moe_down_fwd(const void* act, int64_t I, const int32_t* 
   g.ovl = overlay;
   g.ovl_words = overlay_words;
   const int64_t max_tiles = (S / NK_BM + E) * ((H + NK_BN - 1) / NK_BN);
-  return launch_gemm_nk<EPI_STORE>(g, dtype, max_tiles, S, as_stream(stream), "moe_down_fwd");
+  return launch_gemm_nk<EPI_STORE>(g, dtype, max_tiles, S, S, as_stream(stream), "moe_down_fwd");
 }
 
 // Forward gate_up + SwiGLU with dense weights held in a slot arena (usaf_amd's
@@ -2349,7 +2239,7 @@ extern "C" int usaf_hip_moe_gate_up_fwd_slots(const void* x, int64_t T_rows, int
     return set_error(USAF_ERR_UNSUPPORTED, "moe_gate_up_fwd_slots: the fragment-order arena needs 16-byte aligned "
                                            "activation rows, H %% 128 == 0, E <= %d and blocks below 4 GiB", Q_MAX_E);
   const int64_t max_tiles = (S / NK_BM + E) * ((I + 127) / 128);
-  return launch_gemm_nk<EPI_SWIGLU_FWD>(g, dtype, max_tiles, T_rows, as_stream(stream), "moe_gate_up_fwd_slots");
+  return launch_gemm_nk<EPI_SWIGLU_FWD>(g, dtype, max_tiles, S, T_rows, as_stream(stream), "moe_gate_up_fwd_slots");
 }
 
 // Forward down projection with dense weights in a slot arena [n_slots, H, I].
@@ -2373,7 +2263,7 @@ extern "C" int usaf_hip_moe_down_fwd_slots(const void* act, int64_t I, const int
     return set_error(USAF_ERR_UNSUPPORTED, "moe_down_fwd_slots: the fragment-order arena needs 16-byte aligned "
                                            "activation rows, I %% 128 == 0, E <= %d and blocks below 4 GiB", Q_MAX_E);
   const int64_t max_tiles = (S / NK_BM + E) * ((H + NK_BN - 1) / NK_BN);
-  return launch_gemm_nk<EPI_STORE>(g, dtype, max_tiles, S, as_stream(stream), "moe_down_fwd_slots");
+  return launch_gemm_nk<EPI_STORE>(g, dtype, max_tiles, S, S, as_stream(stream), "moe_down_fwd_slots");
 }
 
 // Backward through the down projection and SwiGLU: dgu[m] from dcur[m] @ W_down[e].
@@ -2432,7 +2322,7 @@ extern "C" int usaf_hip_moe_down_bwd_t(const void* dcur, int64_t H, const void* 
   g.ovl = overlay;
   g.ovl_words = overlay_words;
   const int64_t max_tiles = (S / Q_BM + E) * ((I + Q_BN - 1) / Q_BN);
-  return launch_q4t<EPI_SWIGLU_BWD>(g, dtype, max_tiles, S, as_stream(stream), "moe_down_bwd_t");
+  return launch_q4t<EPI_SWIGLU_BWD>(g, dtype, max_tiles, S, S, as_stream(stream), "moe_down_bwd_t");
 }
 
 // dx_slots from dgu @ W_gate_up[e] on the transposed copy W_gate_up^T [E, H, 2I].
@@ -2454,5 +2344,5 @@ extern "C" int usaf_hip_moe_gate_up_bwd_t(const void* dgu, int64_t I, const int3
   g.ovl = overlay;
   g.ovl_words = overlay_words;
   const int64_t max_tiles = (S / Q_BM + E) * ((H + Q_BN - 1) / Q_BN);
-  return launch_q4t<EPI_STORE>(g, dtype, max_tiles, S, as_stream(stream), "moe_gate_up_bwd_t");
+  return launch_q4t<EPI_STORE>(g, dtype, max_tiles, S, S, as_stream(stream), "moe_gate_up_bwd_t");
 }
