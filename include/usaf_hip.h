@@ -187,6 +187,17 @@ int usaf_hip_router_fwd(const void* x, const void* w, int64_t T, int64_t E, int6
                         void* stream);
 
 /*
+ * Dense weight gradient of the routed experts (autograd of the reference's
+ * trainable experts, usaf/olmoe_dml.py:22-31):
+ *   out[e, r, c] = out_dtype( sum_{s in [offsets[e], offsets[e+1])} fp32(dy[s, r]) * fp32(x[row(s), c]) )
+ * for every expert, zeros for one without slots; row(s) = x_rows ? x_rows[s] : s.
+ * dy [S, R] and x [*, C] row-major 16-bit (dtype), fp32 accumulation, out
+ * [E, R, C] in fp32, fp16 or bf16.  R and C multiples of 8, 16-byte aligned operands.
+ */
+int usaf_hip_moe_weight_grad(const void* dy, const void* x, const int32_t* x_rows, const int32_t* offsets, int64_t E,
+                             int64_t R, int64_t C, int32_t dtype, void* out, int32_t out_dtype, void* stream);
+
+/*
  * Weight gradient of the router's linear layer (autograd of qwen3moe_dml.py:72,
  * router_logits = F.linear(hs, router.weight)):
  *   dw[e, h] = dtype( sum_t fp32(dlogits[t, e]) * fp32(x[t, h]) )      [E, H]

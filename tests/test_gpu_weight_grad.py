@@ -1,0 +1,40 @@
+"""Dense expert weight gradients (usaf_hip_moe_weight_grad) where its tiles end:
+experts without slots, with 1, 63, 64, 65 and 130, rows and columns that are not
+whole 128 x 128 tiles, expert counts that do and do not divide over the dies,
+gathered and plain rows.  Operands are integers in [-4, 4]: the sums are exact in
+fp32, so every output type must hold the 64-bit product rounded once, bit for bit.
+"""
+import pytest
+import torch
+
+from usaf_amd import _native as N
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("E,R,C,counts,dt,out_dt,gathered", [
+    (5, 136, 72, [0, 1, 65, 64, 130], torch.bfloat16, torch.bfloat16, True),
+    (8, 256, 128, [63, 0, 2], torch.float16, torch.float16, False),
+    (16, 128, 264, [7, 128], torch.bfloat16, torch.float32, True),
+    (3, 8, 8, [1, 0, 9], torch.float16, torch.float32, False),
+    (8, 128, 128, [0], torch.bfloat16, torch.bfloat16, False),
+])
+def test_weight_grad(gpu_device, E, R, C, counts, dt, out_dt, gathered):
+    gen = torch.Generator().manual_seed(E + R + C)
+    counts = [counts[e % len(counts)] for e in range(E)]
+    S, T = sum(counts), 50
+    print(f"[gpu-case] weight grad E={E} R={R} C={C} S={S} {dt} -> {out_dt} gathered={gathered}", flush=True)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    dy = torch.randint(-4, 5, (max(S, 1), R), generator=gen).to(dt)
+    x = torch.randint(-4, 5, (T if gathered else max(S, 1), C), generator=gen).to(dt)
+    rows = torch.randint(0, T, (max(S, 1),), generator=gen).to(torch.int32) if gathered else None
+    d = lambda t: None if t is None else t.to(gpu_device)
+    ddy, dx, drows, doffs = d(dy), d(x), d(rows), d(offs)
+    out = torch.full((E, R, C), float("nan"), dtype=out_dt, device=gpu_device)
+    N.call("usaf_hip_moe_weight_grad", ddy.data_ptr(), dx.data_ptr(), N.ptr(drows), doffs.data_ptr(), E, R, C,
+           N.dtype_code(dt), out.data_ptr(), N.dtype_code(out_dt), N.stream_ptr(gpu_device))
+    torch.cuda.synchronize()
+    xs = x if rows is None else x[rows.long()]
+    for e in range(E):
+        a, b = int(offs[e]), int(offs[e + 1])
+        assert torch.equal(out[e].cpu(), (dy[a:b].double().t() @ xs[a:b].double()).to(out_dt)), e

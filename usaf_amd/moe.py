@@ -548,9 +548,10 @@ class RoutedExpertsFn(torch.autograd.Function):
         code = N.dtype_code(dt)
         dweights = torch.zeros(T, E, dtype=dt, device=dev)
         want_gu, want_dn = ctx.needs_input_grad[4], ctx.needs_input_grad[5]
-        d_wgu = torch.zeros(E, 2 * I, H, dtype=ctx.wdt[0], device=dev) if want_gu else None
-        d_wdn = torch.zeros(E, H, I, dtype=ctx.wdt[1], device=dev) if want_dn else None
+        d_wgu = d_wdn = None
         if S == 0:
+            d_wgu = torch.zeros(E, 2 * I, H, dtype=ctx.wdt[0], device=dev) if want_gu else None
+            d_wdn = torch.zeros(E, H, I, dtype=ctx.wdt[1], device=dev) if want_dn else None
             return torch.zeros_like(hs), dweights, None, None, d_wgu, d_wdn, None
         dcur = torch.empty(S, H, dtype=dt, device=dev)
         dcur_blk = None
@@ -583,7 +584,7 @@ class RoutedExpertsFn(torch.autograd.Function):
             _capture(capture, "down_proj", dcur, act, None, b, (E, H, I), dt, dy_blocked=dcur_blk,
                      x_blocked=ctx.act_blk)
         if want_dn:
-            _dense_weight_grad(d_wdn, dcur, act, None, b)
+            d_wdn = _dense_weight_grad(dcur, act, None, b, ctx.wdt[1])
         dx_slots = torch.empty(S, H, dtype=dt, device=dev)
         tq = ew._ptrs_t("gate_up")
         if tq is not None:
@@ -601,7 +602,7 @@ class RoutedExpertsFn(torch.autograd.Function):
         if capture is not None:
             _capture(capture, "gate_up_proj", dgu, hs, b.token_idx, b, (E, 2 * I, H), dt)
         if want_gu:
-            _dense_weight_grad(d_wgu, dgu, hs, b.token_idx, b)
+            d_wgu = _dense_weight_grad(dgu, hs, b.token_idx, b, ctx.wdt[0])
         if ctx.link is not None and dweights is not None:
             # the router's backward (next, it needs dweights) adds its grad-input to
             # this one in the same kernel: one sum instead of autograd's extra add
@@ -616,18 +617,19 @@ def _no_overlay(ew: ExpertWeights, which: str) -> None:
                                   f"(E <= {_T_MAX_E}, rows % 64 == 0 and the GEMM's N, K multiples of 128)")
 
 
-def _dense_weight_grad(out: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, x_rows: Optional[torch.Tensor],
-                       b: "Buckets") -> None:
-    """out[e] = dy_e^T @ x_e for every expert with slots (fp32 products, stored in
-    out's dtype): the dense expert-weight gradient autograd gives the reference's
-    trainable experts (olmoe_dml.py:22-31, olmoe_streaming.py:91-97)."""
-    offs = b.offsets.tolist()
-    for ei in range(len(offs) - 1):
-        s0, s1 = offs[ei], offs[ei + 1]
-        if s0 == s1:
-            continue
-        xe = x.index_select(0, x_rows[s0:s1].long()) if x_rows is not None else x[s0:s1]
-        out[ei] = torch.mm(dy[s0:s1].t().float(), xe.float()).to(out.dtype)
+def _dense_weight_grad(dy: torch.Tensor, x: torch.Tensor, x_rows: Optional[torch.Tensor], b: "Buckets",
+                       out_dtype: torch.dtype) -> torch.Tensor:
+    """[E, R, C] dy_e^T @ x_e of every expert's slots (zeros without slots; fp32
+    sums, stored in out_dtype): the dense expert-weight gradient autograd gives the
+    reference's trainable experts (olmoe_dml.py:22-31, olmoe_streaming.py:91-97)."""
+    E, R, C = b.offsets.numel() - 1, dy.shape[1], x.shape[1]
+    kernel_dtype = out_dtype if out_dtype in (torch.float16, torch.bfloat16) else torch.float32
+    out = torch.empty(E, R, C, dtype=kernel_dtype, device=dy.device)
+    if x.data_ptr() % 16:  # a view that starts inside a 16-byte piece
+        x = x.clone()
+    N.call("usaf_hip_moe_weight_grad", dy.data_ptr(), x.data_ptr(), N.ptr(x_rows), b.offsets.data_ptr(), E, R, C,
+           N.dtype_code(dy.dtype), out.data_ptr(), N.dtype_code(kernel_dtype), N.stream_ptr(dy.device))
+    return out.to(out_dtype)
 
 
 @dataclass
