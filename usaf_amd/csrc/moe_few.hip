@@ -42,47 +42,6 @@ constexpr int FEW_SLOTS = 32;  // slots of an m-tile: one MFMA column block
 constexpr int FEW_XCDS = 8;    // accelerator dies, blocks dispatched round-robin over them
 constexpr int FEW_IMG = 4 * 1024 + 128;  // overlay: four fragment images and 128 bytes of discards
 
-// m-tile mt of the list (experts in order, each in tiles of FEW_SLOTS) -> expert,
-// first slot, slots; false past the end.  One wave, offsets from global
-// memory: lane l counts the tiles of experts 4 l .. 4 l + 3 (E <= 255).
-__device__ __forceinline__ bool few_tile(const GemmArgs& g, int lane, int mt, int& e, int& m_beg, int& valid) {
-  int off[5], c[4], sum = 0;
-#pragma unroll
-  for (int k = 0; k < 5; ++k) {
-    const int i = 4 * lane + k;
-    off[k] = g.offsets[i < g.E ? i : g.E];
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    c[k] = (off[k + 1] - off[k] + FEW_SLOTS - 1) / FEW_SLOTS;
-    sum += c[k];
-  }
-  int incl = sum;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int o = __shfl_up(incl, d, 64);
-    if (lane >= d) incl += o;
-  }
-  const uint64_t past = __ballot(incl > mt);  // lanes at or after the owner
-  if (past == 0) return false;
-  const int src = __builtin_ctzll(past);
-  int j = mt - (incl - sum), ee = 4 * lane, beg = off[0], end = off[1];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    if (ee == 4 * lane + k && j >= c[k]) {  // past expert 4 l + k
-      j -= c[k];
-      ee = 4 * lane + k + 1;
-      beg = off[k + 1];
-      end = off[k + 2];
-    }
-  }
-  e = __builtin_amdgcn_readlane(ee, src);
-  m_beg = __builtin_amdgcn_readlane(beg + j * FEW_SLOTS, src);
-  const int rem = __builtin_amdgcn_readlane(end, src) - m_beg;
-  valid = rem < FEW_SLOTS ? rem : FEW_SLOTS;
-  return true;
-}
-
 // One wave's LDS: activation tiles and overlay images, at the end its partial tile.
 template <int NU, bool OVL>
 constexpr int few_wave_lds() {
@@ -367,7 +326,7 @@ __global__ __launch_bounds__(FEW_THREADS, WPS) void moe_few_kernel(const GemmArg
   const int mt = grp / chunks, sub = wave / ks, part = wave - sub * ks;
   FewTile t;
   t.b = ((grp - mt * chunks) * per + (int)blockIdx.x / FEW_XCDS % per) * (FEW_WAVES / ks) + sub;
-  if (!few_tile(g, lane, mt, t.e, t.m_beg, t.valid)) return;  // block-uniform
+  if (!slot_tile<FEW_SLOTS>(g, lane, mt, t.e, t.m_beg, t.valid)) return;  // block-uniform
   // waves past the weight's rows: all ks of a group together
   if ((int64_t)t.b * (EPI == EPI_SWIGLU_FWD ? 16 : 32) * NU >= g.N) return;
   few_tile_run<NU, EPI, DT, BT, OVL>(g, t, sm, wave, lane, ks, part);

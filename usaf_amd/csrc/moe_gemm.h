@@ -44,6 +44,11 @@ struct GemmArgs {
 bool few_slots(const GemmArgs& g, int epi, bool transposed, int64_t S);
 int launch_few(const GemmArgs& g, int epi, bool transposed, int dt, int64_t S, hipStream_t st, const char* what);
 
+// Dense weights and short m-tiles (moe_dense.hip): whether a GEMM over S slots
+// goes to that kernel, and its launch.  kn: the weight is [K, N] (grad-input).
+bool dense_slots(const GemmArgs& g, int epi, bool kn, int64_t S, int64_t a_rows_total);
+int launch_dense(const GemmArgs& g, int epi, bool kn, int dt, int64_t S, hipStream_t st, const char* what);
+
 namespace {
 
 // Workgroup barrier ordering LDS accesses only.  __syncthreads() also orders
@@ -63,6 +68,48 @@ __device__ __forceinline__ int64_t weight_block(const GemmArgs& g, int e) {
   if (g.w_slot == nullptr) return e;
   const int64_t s = g.w_slot[e];
   return s < 0 ? 0 : (s >= g.n_slots ? g.n_slots - 1 : s);
+}
+
+// m-tile mt of the list (experts in order, each in tiles of SLOTS) -> expert,
+// first slot, slots; false past the end.  One wave, offsets from global
+// memory: lane l counts the tiles of experts 4 l .. 4 l + 3 (E <= 255).
+template <int SLOTS>
+__device__ __forceinline__ bool slot_tile(const GemmArgs& g, int lane, int mt, int& e, int& m_beg, int& valid) {
+  int off[5], c[4], sum = 0;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    const int i = 4 * lane + k;
+    off[k] = g.offsets[i < g.E ? i : g.E];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    c[k] = (off[k + 1] - off[k] + SLOTS - 1) / SLOTS;
+    sum += c[k];
+  }
+  int incl = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += o;
+  }
+  const uint64_t past = __ballot(incl > mt);  // lanes at or after the owner
+  if (past == 0) return false;
+  const int src = __builtin_ctzll(past);
+  int j = mt - (incl - sum), ee = 4 * lane, beg = off[0], end = off[1];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    if (ee == 4 * lane + k && j >= c[k]) {  // past expert 4 l + k
+      j -= c[k];
+      ee = 4 * lane + k + 1;
+      beg = off[k + 1];
+      end = off[k + 2];
+    }
+  }
+  e = __builtin_amdgcn_readlane(ee, src);
+  m_beg = __builtin_amdgcn_readlane(beg + j * SLOTS, src);
+  const int rem = __builtin_amdgcn_readlane(end, src) - m_beg;
+  valid = rem < SLOTS ? rem : SLOTS;
+  return true;
 }
 
 __device__ __forceinline__ uint32_t h2_to_bf2(uint32_t h2) {

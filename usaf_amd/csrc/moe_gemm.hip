@@ -2059,6 +2059,7 @@ int launch_gemm_nk(const GemmArgs& g, int dt, int64_t max_tiles, int64_t S, int6
   if (int rc = check_ovl(g, EPI, what)) return rc;
   if (dma && few_slots(g, EPI, false, S)) return launch_few(g, EPI, false, dt, S, st, what);
   const bool dw = dense && dw_dma_ok(g, a_rows_total);
+  if (dw && dense_slots(g, EPI, false, S, a_rows_total)) return launch_dense(g, EPI, false, dt, S, st, what);
   int rc;
   if (dt == USAF_BF16)
     rc = dw ? launch_dw_one<EPI, USAF_BF16>(g, (unsigned)blocks, st)
@@ -2091,7 +2092,7 @@ int launch_one(const GemmArgs& g, unsigned blocks, hipStream_t st) {
 
 template <int BMODE, int EPI>
 int launch_gemm(const GemmArgs& g, int dt, int64_t max_tiles, int64_t a_rows_total, hipStream_t st,
-                const char* what) {
+                const char* what) {  // one A row per slot: a_rows_total slots
   // activation offsets are 32-bit inside the kernel
   if (a_rows_total * g.lda >= ((int64_t)1 << 31))
     return set_error(USAF_ERR_UNSUPPORTED, "%s: activation operand of %lld x %lld elements exceeds 2^31", what,
@@ -2100,6 +2101,8 @@ int launch_gemm(const GemmArgs& g, int dt, int64_t max_tiles, int64_t a_rows_tot
   if (blocks > max_tiles) blocks = max_tiles;
   if (blocks < 1) blocks = 1;
   const bool dense = g.w16 != nullptr;
+  if (dense && dense_slots(g, EPI, true, a_rows_total, a_rows_total))
+    return launch_dense(g, EPI, true, dt, a_rows_total, st, what);
   int rc;
   if (dt == USAF_BF16)
     rc = dense ? launch_one<BMODE, EPI, BQ_DENSE16, USAF_BF16>(g, (unsigned)blocks, st)
