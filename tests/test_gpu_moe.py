@@ -1099,3 +1099,22 @@ def test_router_fwd_exact_logits(gpu_device, T, E, H, k, norm):
     assert torch.equal(weights.cpu() != 0, w_ref != 0), "routing mask differs from the oracle"
     assert torch.equal(weights.cpu().view(torch.int16), w2.cpu().view(torch.int16))
     assert torch.equal(probs.cpu(), p2.cpu())
+
+
+@pytest.mark.parametrize("dense", [False, True])
+@pytest.mark.parametrize("T", [0, 5])
+def test_experts_no_routed_pair(gpu_device, T, dense):
+    """No tokens, or tokens without any routed expert: zeros forward and zero
+    gradients backward, as the reference's loop over experts that got no token."""
+    _say(f"experts fwd+bwd without a routed pair, T={T} dense={dense}")
+    E, H, I, dt = 4, 256, 128, torch.bfloat16
+    L = make_layer(gpu_device, E, H, I, 1, 1, dt, seed=5, dense=dense)
+    hs = torch.ones(T, H, dtype=dt, device=gpu_device, requires_grad=True)
+    w = torch.zeros(T, E, dtype=dt, device=gpu_device, requires_grad=True)
+    params = (L["ew"].gate_up.requires_grad_(True), L["ew"].down.requires_grad_(True)) if dense else None
+    out = G.routed_experts(hs, w, L["ew"], weight_params=params)
+    out.backward(torch.ones_like(out))
+    torch.cuda.synchronize()
+    for t in (out, hs.grad, w.grad, *([p.grad for p in params] if dense else [])):
+        assert t is not None and not t.any()
+    assert out.shape == hs.shape and (not dense or params[0].grad.shape == params[0].shape)

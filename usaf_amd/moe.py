@@ -524,7 +524,7 @@ class RoutedExpertsFn(torch.autograd.Function):
             q, sz, w16 = ew._ptrs("down", dt)
             timed_call("usaf_hip_moe_down_fwd", act.data_ptr(), I, b.offsets.data_ptr(), S, E, H, q, sz, w16,
                        code, y.data_ptr(), *ew._ovl("down_fwd", dt), st)
-        out = combine(y, weights, b.pair_slot, dt)
+        out = combine(y, weights, b.pair_slot, dt) if S > 0 else torch.zeros_like(hs)
         ctx.ew = ew
         ctx.capture = capture
         ctx.link = link
@@ -552,7 +552,7 @@ class RoutedExpertsFn(torch.autograd.Function):
         if S == 0:
             d_wgu = torch.zeros(E, 2 * I, H, dtype=ctx.wdt[0], device=dev) if want_gu else None
             d_wdn = torch.zeros(E, H, I, dtype=ctx.wdt[1], device=dev) if want_dn else None
-            return torch.zeros_like(hs), dweights, None, None, d_wgu, d_wdn, None
+            return torch.zeros_like(hs), dweights, None, None, d_wgu, d_wdn, None, None
         dcur = torch.empty(S, H, dtype=dt, device=dev)
         dcur_blk = None
         if _sampled_blocked(capture, b) and _blocked_ok(dout) and _blocked_ok(y):
