@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from usaf_amd import _native as N
+from usaf_amd import moe as G
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +39,24 @@ def test_weight_grad(gpu_device, E, R, C, counts, dt, out_dt, gathered):
     for e in range(E):
         a, b = int(offs[e]), int(offs[e + 1])
         assert torch.equal(out[e].cpu(), (dy[a:b].double().t() @ xs[a:b].double()).to(out_dt)), e
+
+
+def test_weight_grad_of_saved_tensors_in_another_layout(gpu_device):
+    """A saved-tensor hook may hand the activations back in another memory order."""
+    print("[gpu-case] weight grad with saved hidden states and activations as transposed views", flush=True)
+    gen = torch.Generator().manual_seed(1)
+    E, H, I, T, dt = 4, 256, 128, 40, torch.bfloat16
+    d = lambda *s: (torch.randn(s, generator=gen) * 0.1).to(dt).to(gpu_device)
+    hs, dout, wg, wd = d(T, H), d(T, H), d(E, 2 * I, H), d(E, H, I)
+    w = (torch.rand(T, E, generator=gen) * (torch.rand(T, E, generator=gen) < 0.5)).to(dt).to(gpu_device)
+    grads = []
+    # hs [T, H] and act [S, I]; gu and y as they are
+    turn = lambda t: t.t().contiguous().t() if t.shape[1] == I or t.shape[0] == T else t
+    for unpack in (lambda t: t, turn):
+        p = [wg.clone().requires_grad_(True), wd.clone().requires_grad_(True)]
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            out = G.routed_experts(hs.clone().requires_grad_(True), w, G.ExpertWeights(*p), weight_params=tuple(p))
+        out.backward(dout)
+        torch.cuda.synchronize()
+        grads.append([q.grad for q in p])
+    assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])

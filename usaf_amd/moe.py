@@ -625,6 +625,7 @@ def _dense_weight_grad(dy: torch.Tensor, x: torch.Tensor, x_rows: Optional[torch
     E, R, C = b.offsets.numel() - 1, dy.shape[1], x.shape[1]
     kernel_dtype = out_dtype if out_dtype in (torch.float16, torch.bfloat16) else torch.float32
     out = torch.empty(E, R, C, dtype=kernel_dtype, device=dy.device)
+    x = x.contiguous()  # a saved-tensor hook may have changed its layout
     if x.data_ptr() % 16:  # a view that starts inside a 16-byte piece
         x = x.clone()
     N.call("usaf_hip_moe_weight_grad", dy.data_ptr(), x.data_ptr(), N.ptr(x_rows), b.offsets.data_ptr(), E, R, C,
