@@ -1,7 +1,7 @@
 """The grouped 4-bit GEMMs at few slots per expert (moe_few.hip), where their
 tiles end: experts without slots, with 1, 31, 32, 33 and 65, one expert only,
-255 experts, widths that leave waves without rows, every split of the
-contraction.
+255 experts, widths that leave waves without rows (unsplit and split in two),
+every split of the contraction, four weight-row units a wave.
 
 Weights and activations are small integers (scale 1, zero -8; activations in
 [-2, 2]), so every sum is exact in fp32 in any order and the outputs that are
@@ -41,6 +41,7 @@ CASES = [  # E, H, I, slots of the experts in turn, dtype, overlay
     (128, 2048, 768, [16, 9, 33, 2], torch.bfloat16, True),
     (128, 2048, 768, [16, 30, 0], torch.float16, False),
     (2, 4096, 384, [19, 1], torch.bfloat16, False),
+    (128, 640, 896, [16, 9, 33, 2], torch.bfloat16, False),  # down, d(act): unsplit blocks with two idle waves
 ]
 
 
@@ -108,3 +109,42 @@ def test_few_slots(gpu_device, E, H, I, slots, dt, overlay):
     da, sig = exact(dcur, wd, False).double(), torch.sigmoid(g)
     assert close(dgu.cpu(), torch.cat([da * u * sig * (1 + g * (1 - sig)), da * g * sig], 1),
                  torch.cat([(da * u).abs(), (da * g).abs()], 1))
+
+
+@pytest.mark.parametrize("gemm,E,cols,K,slots", [
+    ("gate_up", 255, 160, 1536, [1, 0, 3]),  # split in two: the last block's second pair of waves has no rows
+    ("gate_up", 8, 3008, 3072, [28, 33, 20]),  # four units a wave, split in four
+    ("down", 8, 6016, 3072, [28, 33, 20]),
+])
+def test_few_slots_one_gemm(gpu_device, gemm, E, cols, K, slots):
+    """cols columns from a contraction of K (gate_up: cols gate and cols up rows)."""
+    dev, dt = gpu_device, torch.bfloat16
+    gen = torch.Generator().manual_seed(E + cols + K)
+    counts = [slots[e % len(slots)] for e in range(E)]
+    S, rows = sum(counts), 2 * cols if gemm == "gate_up" else cols
+    assert 0 < S <= 28 * E
+    print(f"[gpu-case] few slots {gemm} E={E} cols={cols} K={K} S={S}", flush=True)
+    q = torch.randint(-128, 128, (E, rows * K // 2), generator=gen, dtype=torch.int8)
+    one = torch.ones(E * rows * K // 128, dtype=torch.float16)
+    w = G.Q4Tensor(q.view(-1, 64).to(dev), one.to(dev), (-8 * one).to(dev), torch.Size((E, rows, K)), 128)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    x = torch.randint(-2, 3, (S, K), generator=gen).to(dt)
+    d_x, d_offs, d_rows = x.to(dev), offs.to(dev), torch.arange(S, dtype=torch.int32, device=dev)
+    out = torch.full((S, rows), float("nan"), dtype=dt, device=dev)
+    code, st = N.dtype_code(dt), N.stream_ptr(dev)
+    if gemm == "gate_up":
+        act = torch.empty(S, cols, dtype=dt, device=dev)
+        N.call("usaf_hip_moe_gate_up_fwd", d_x.data_ptr(), S, K, d_rows.data_ptr(), d_offs.data_ptr(), S, E, cols,
+               w.q.data_ptr(), w.scale_zero().data_ptr(), None, code, out.data_ptr(), act.data_ptr(), None, None,
+               None, 0, st)
+    else:
+        N.call("usaf_hip_moe_down_fwd", d_x.data_ptr(), K, d_offs.data_ptr(), S, E, cols, w.q.data_ptr(),
+               w.scale_zero().data_ptr(), None, code, out.data_ptr(), None, 0, st)
+    torch.cuda.synchronize()
+    got = out.cpu()
+    for e in range(E):
+        a, b = int(offs[e]), int(offs[e + 1])
+        if a < b:
+            raw = q[e].view(torch.uint8)
+            vals = torch.stack([raw & 15, raw >> 4], 1).double().view(rows, K) - 8
+            assert torch.equal(got[a:b], (x[a:b].double() @ vals.t()).to(dt)), e

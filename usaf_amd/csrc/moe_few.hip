@@ -22,16 +22,16 @@
 //   k = 32 h + 8 j + [0, 8) of row l32 in register j -- so the overlay tables
 //   serve both kernels.
 //
-// What bounds it: the dequantization.  All 128 experts of a Qwen3 layer's gate_up
-// are 25 M wave instructions in bf16 (8 a pair of weights), 43 us of the VALU,
-// against 33 us for reading the 214 MB of codes at the 6.5 TB/s a plain read
-// reaches here.  Measured (Qwen3 layer, us, gate_up / down / d(act) / d(x); before:
-// moe_gemm_q4_kernel):
-//   1 token, bf16      36 / 17            -> 10.6 / 7.3
-//   24 tokens          111 / 57           -> 70 / 35
-//   333 tokens         119 / 63 / 76 / 114 -> 79 / 43 / 56 / 81
-//   256, fp16, overlay 148 / 75 / 88 / 134 -> 108 / 56 / 73 / 112
-// and 302 / 257 -> 190 / 100 for 40 tokens of a Mixtral layer.
+// What bounds it: the dequantization and, below it, whole rounds of blocks.  All
+// 128 experts of a Qwen3 layer's gate_up are 25 M wave instructions in bf16 (8 a pair
+// of weights), 43 us of the VALU, and 33 us of reading 214 MB at 6.5 TB/s; the 97
+// experts of 24 tokens take 67 us, all 128 at 256 tokens 86.  Measured with cold
+// weights (us, moe_gemm_q4_kernel / this one; gate_up, down, d(act), d(x)):
+//   Qwen3, 24 tokens, bf16       116 / 67, 63 / 41, 78 / 48, 110 / 75
+//   Qwen3, 320 tokens, bf16      119 / 88, 66 / 48, 81 / 54, 115 / 85
+//   Qwen3, 256, fp16, overlay    136 / 103, 73 / 58, 89 / 72, 134 / 110
+//   Mixtral, 40 tokens, bf16     311 / 182, 265 / 101, 138 / 99, 431 / 173
+// and one token, warm, 36 / 10.6, 17 / 7.3.
 #include "moe_gemm.h"
 
 namespace usaf {
@@ -345,25 +345,38 @@ void launch_few_one(const GemmArgs& g, int64_t S, int ks, hipStream_t st) {
       <<<(unsigned)blocks, FEW_THREADS, 0, st>>>(g, (int)per, (int)chunks, ks);
 }
 
-// NU and the split ks of the contraction.
+// NU and the split ks of the contraction (cold weights, us).
 // * ks: six groups a wave or more, so that its prologue (the m-tile, the first
 //   codes: about 3 us) is a small part of it; but four where even that leaves the
 //   1,024 SIMDs short of two waves (one token: 10.6 us split four ways, 26 unsplit).
-// * NU = 4 reads the activations half as often as NU = 2 and is the faster one
-//   wherever its 190 to 256 registers leave enough waves: measured 79.6 against
-//   87 us for gate_up of 333 tokens at ks = 2, 186 against 192 for Mixtral's at
-//   ks = 4.  At ks = 1 (K = 768: 44 against 48 us) and with an overlay (106
-//   against 112 us) two units at three waves a SIMD hide more; a transposed
-//   weight's scale words are shared by the units and want four.
+// * NU = 2 keeps three or four blocks a CU (two with a transposed weight) and halves
+//   what a last, partly filled round costs against NU = 4.  NU = 4 reads the activations
+//   half as often, and a transposed weight's scale words, which its units share.
+//   Forward, NU = 4 / 2: gate_up at ks = 2 79 / 67 (24 tokens, Qwen3), 86 / 86 (256), 80 / 72
+//   (160, OLMoE, Zipf(1.1)); with the contraction split four ways equal, 182 / 183 (40,
+//   Mixtral), and 5 % faster with warm weights.
+// * Transposed: NU = 4 needs two full rounds of blocks.  Qwen3 d(x), 1,024 blocks: 84 / 91,
+//   Zipf(1.1) 98 / 106; OLMoE d(x), 512 blocks: 58 / 62, but 77 / 72.  With
+//   an overlay it takes all 256 registers and spills four (20 bytes a lane).
+// * An overlay keeps every wave longer.  Where NU = 2 does not fill two rounds either,
+//   ks = 4 evens them out: OLMoE d(act), ks = 2 / 4, 47 / 51, Zipf(1.1) 69 / 61, Qwen3 71 / 72, 84 / 88.
 template <int EPI, int DT, bool BT, bool OVL>
 void launch_few_dt(const GemmArgs& g, int64_t S, hipStream_t st) {
   const int64_t unit = EPI == EPI_SWIGLU_FWD ? 16 : 32, groups = g.K / 128;
   const int64_t tiles = (S < g.E ? S : g.E) + S / (2 * FEW_SLOTS);  // about as many m-tiles as there will be
   const bool few = tiles * (g.N / (4 * unit)) * 4 < 2048;
-  const int ks = few || groups >= 24 ? 4 : groups >= 12 ? 2 : 1;
-  const bool wide = !few && g.N % (4 * unit) == 0 && (BT || (ks > 1 && !OVL));
-  if (wide) launch_few_one<4, 2, EPI, DT, BT, OVL>(g, S, ks, st);
-  else launch_few_one<2, BT ? 2 : 3, EPI, DT, BT, OVL>(g, S, ks, st);
+  int ks = few || groups >= 24 ? 4 : groups >= 12 ? 2 : 1;
+  bool wide = !few && ks == 4;
+  if constexpr (BT) {
+    // waves' units of an m-tile for each used expert, against two rounds of two blocks a CU
+    const int64_t units = (S < g.E ? S : g.E) * (g.N / 32), two = 4 * (int64_t)device_cu_count() * FEW_WAVES;
+    wide = units * ks >= two * 4;
+    if (OVL && units * ks < two * 2) ks = 4;
+  }
+  if constexpr (BT || !OVL) {
+    if (wide && g.N % (4 * unit) == 0) return launch_few_one<4, 2, EPI, DT, BT, OVL>(g, S, ks, st);
+  }
+  launch_few_one<2, BT ? 2 : 3, EPI, DT, BT, OVL>(g, S, ks, st);
 }
 
 template <int EPI, bool BT>
@@ -382,15 +395,30 @@ int launch_few_epi(const GemmArgs& g, int dt, int64_t S, hipStream_t st, const c
 
 }  // namespace
 
-// The line against moe_gemm_q4_kernel, in slots per expert on average.  Past 32
+// The lines against moe_gemm_q4_kernel, in slots per expert on average.  Past 32
 // slots an expert takes a second m-tile and its codes are dequantized again; with
-// a random routing that begins at an average of about 20.  Measured at Qwen3 (us,
-// that kernel / this one): forward at 28: 188 / 152, at 32: 188 / 178 (with an
-// overlay 233 / 207, 227 / 226); backward at 21: 191 / 138, at 24: 192 / 168,
-// with an overlay at 16: 222 / 185, at 24: 222 / 250.
+// a random routing that begins at an average of about 20.  Measured with cold
+// weights at the lines (Qwen3 layer, us, that kernel / this one; routings uniform,
+// Zipf(1.1), Zipf(2)):
+// * forward, 28: gate_up 121 / 108, 153 / 117, 130 / 118, down 68 / 58, 83 / 63, 67 / 67.
+// * transposed, 20: d(act) 81 / 54, 86 / 65, 89 / 64, d(x) 114 / 85, 144 / 112, 111 / 95.
+// With an overlay (fp16) the same lines where the other kernel, a tile of 256 rows a
+// CU, leaves half of its last round or more idle.  Where it fills its rounds:
+// * forward 24: at 24 gate_up 139 / 126, 174 / 142, 152 / 137, down 74 / 67, 95 / 75, 74 / 73; at 28
+//   141 / 133, 177 / 145, 151 / 154 and 74 / 68, 94 / 76, 75 / 84.
+// * transposed, a contraction below 24 groups, 20: d(x) at 20 136 / 111, 171 / 149, 133 / 134 (at
+//   16 134 / 110, 143 / 139, 113 / 132); OLMoE d(act) 53 / 52, 65 / 62, 67 / 68.
+// * transposed, a longer one, never: Mixtral d(act) at 16 158 / 141, 161 / 198, 163 / 198.
+// The host does not see the routing: with every token on the same eight of 128
+// experts (448 tokens, 448 slots each) gate_up and down take 74 + 43 us against 60 + 32.
 bool few_slots(const GemmArgs& g, int epi, bool transposed, int64_t S) {
-  const int64_t rows = epi == EPI_SWIGLU_FWD ? 32 : 64;
-  if (S > (transposed ? 20 : 28) * (int64_t)g.E || g.N % rows != 0) return false;
+  const int64_t rows = epi == EPI_SWIGLU_FWD ? 32 : 64, tile = epi == EPI_SWIGLU_FWD ? 128 : 256;
+  int64_t line = transposed ? 20 : 28;
+  if (g.ovl) {
+    const int64_t cus = device_cu_count(), last = (S < g.E ? S : g.E) * ((g.N + tile - 1) / tile) % cus;
+    if (last == 0 || last > cus / 2) line = !transposed ? 24 : g.K >= 24 * 128 ? 0 : 20;
+  }
+  if (S > line * g.E || g.N % rows != 0) return false;
   return (few_m_tiles(g, S) * 2 + FEW_XCDS) * (g.N / rows + 2) < ((int64_t)1 << 30);  // blocks of a launch
 }
 
