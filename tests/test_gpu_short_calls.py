@@ -1,8 +1,8 @@
 """Kernels of short calls at the sizes where they can go wrong: the one-launch
 bucketing (one thread's 64 tokens, one expert, experts that do not divide the
 block, the largest T * E it takes and the next one) and the sampled gradient with
-a thread per position (runs of 0, 16 and more slots, and an average on either
-side of its limit)."""
+a thread per position (runs of 0, 16 and more slots, slices whose average run is
+on either side of its limit, and both kinds in one call)."""
 import pytest
 import torch
 
@@ -41,7 +41,8 @@ def test_bucket_small(gpu_device, T, E, k, dt):
         assert torch.equal(b.pair_slot.cpu(), want)
 
 
-@pytest.mark.parametrize("counts", [[0, 1, 16, 17], [33, 5, 0], [72, 64, 80], [80, 81, 64], [300, 0, 2, 1]])
+@pytest.mark.parametrize("counts", [[0, 1, 16, 17], [33, 5, 0], [72, 64, 80], [80, 81, 64], [300, 0, 2, 1],
+                                    [48, 56, 49], [400, 30, 7, 0, 12, 1, 3, 0, 16]])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_sampled_gradient_short_runs(gpu_device, counts, dt, accumulate):

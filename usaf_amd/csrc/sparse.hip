@@ -405,11 +405,15 @@ __global__ __launch_bounds__(256) void combine_bwd_finish_kernel(const float* __
 // no masking is needed; the position list is cut into one contiguous slice
 // per die, positions sorted by expert keep a die on one expert's operands.
 //
-// SDD_SHORT: up to this many slots per expert on average (padded to 16) a thread
-// takes a whole position instead of a 16-lane group.  Measured on a Qwen3 layer
-// (gate_up + down tensor, us, group / thread): 23 slots 56 + 30 / 20 + 13, 39
-// slots 56 + 33 / 29 + 16, 72 slots 58 + 34 / 52 + 30, 103 slots 58 + 34 / 74 + 42.
-constexpr int SDD_SHORT = 72;
+// SDD_SHORT: a slice whose experts have up to this many (padded) slots on average
+// takes a thread per position instead of a 16-lane group.  The thread form's
+// time grows with that average, the group form's stays until runs pass 128 slots.
+// Measured with cold operands (us, group / thread, gate_up + down tensor), Qwen3: 22
+// slots 65 + 39 / 34 + 21, 51 slots 67 + 41 / 59 + 35, 64 slots 68 + 41 / 73 + 43; OLMoE: 39 slots
+// 47 + 28 / 34 + 21, 63 slots 48 + 29 / 51 + 30.  Each slice decides by itself: under a Zipf
+// routing the slices of the popular experts lose what the average over all hides
+// (OLMoE, 256 tokens, Zipf(1.1), 38 slots: 51 + 32 / 68 + 41).
+constexpr int SDD_SHORT = 56;
 template <int DT>
 __global__ __launch_bounds__(256) void sddmm_blocked_kernel(const uint16_t* __restrict__ rowB,
                                                             const uint16_t* __restrict__ colB,
@@ -420,14 +424,17 @@ __global__ __launch_bounds__(256) void sddmm_blocked_kernel(const uint16_t* __re
                                                             const int64_t* __restrict__ pos_map,
                                                             float* __restrict__ compact, int accumulate) {
   __shared__ int32_t s_pre[BLK_MAX_E + 1];
-  for (int e = threadIdx.x; e <= E; e += blockDim.x) s_pre[e] = table[e];
-  __syncthreads();
   const int gl = threadIdx.x & 15;
   const int dies = gridDim.x < 8 ? (int)gridDim.x : 8;
   const int die = (int)(blockIdx.x % dies);
   const int64_t die_blocks = ((int64_t)gridDim.x + dies - 1 - die) / dies;
   const int64_t lo = n_pos * die / dies, hi = n_pos * (die + 1) / dies;
-  if (s_pre[E] <= SDD_SHORT * E) {
+  // the slice's experts, from its first and last position (sorted by expert)
+  const int ea = lo < hi ? (int)((uint32_t)rcode[lo] >> 21) : 0, eb = lo < hi ? (int)((uint32_t)rcode[hi - 1] >> 21) : 0;
+  for (int e = threadIdx.x; e <= E; e += blockDim.x) s_pre[e] = table[e];
+  __syncthreads();
+  const int e0 = ea < E ? ea : E - 1, e1 = eb < e0 ? e0 : eb < E ? eb : E - 1;
+  if (s_pre[e1 + 1] - s_pre[e0] <= SDD_SHORT * (e1 - e0 + 1)) {
     // Short runs (few slots per expert): a thread per position.  Of a 16-lane
     // group only ld / 8 lanes would have operands, two of them at 16 slots.
     const int64_t n_thr = die_blocks * blockDim.x;
