@@ -1,6 +1,6 @@
 """Kernels of short calls at the sizes where they can go wrong: the one-launch
-bucketing (one thread's 64 tokens, one expert, experts that do not divide the
-block, the largest T * E it takes and the next one) and the sampled gradient with
+bucketing (one thread's 16 tokens, one expert, experts that do not divide the
+block, the most tokens it takes and the next one) and the sampled gradient with
 a thread per position (runs of 0, 16 and more slots, slices whose average run is
 on either side of its limit, and both kinds in one call)."""
 import pytest
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,E,k", [(1, 1, 1), (64, 1, 1), (65, 1, 1), (1, 128, 8), (17, 12, 3), (192, 128, 8),
-                                   (193, 128, 8), (64, 384, 5), (24, 1000, 2), (3072, 8, 2), (63, 48, 48)])
+                                   (193, 128, 8), (64, 384, 5), (24, 1000, 2), (3072, 8, 2), (63, 48, 48),
+                                   (128, 128, 8), (129, 128, 8), (1024, 8, 2), (1025, 8, 2), (16, 1000, 4), (1024, 1, 1)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
 def test_bucket_small(gpu_device, T, E, k, dt):
     print(f"[gpu-case] bucket T={T} E={E} k={k} {dt}", flush=True)

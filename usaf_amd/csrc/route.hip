@@ -309,12 +309,12 @@ __global__ __launch_bounds__(256) void bucket_fill_kernel(const void* __restrict
 
 // The three passes in one block for small [T, E]: three dependent launches of a
 // few microseconds each are most of a short call's bucketing.  Thread (e, seg)
-// holds which of its up to 64 tokens select expert e as a 64-bit mask, so the
-// weights are read once and only the selected ones again.  Measured (T x E, us,
-// three launches / one): 1 x 128 8.7 / 3.7, 24 x 128 11.6 / 4.7, 128 x 128 13.8 /
-// 8.8, 256 x 128 13.9 / 14.5, 1000 x 8 14.6 / 11.1.
-constexpr int kSmallTokens = 64;        // tokens of one thread
-constexpr int64_t kSmallPairs = 24576;  // T * E: past this one CU's reads and writes cost more than the launches
+// holds the weights of its up to 16 tokens for expert e, so they are read once.
+// The line is the tokens of a thread: one CU's serial reads and writes grow with
+// them.  Measured (T x E, cold, us, three launches / one): 1 x 128 14 / 6, 24 x 128
+// 19 / 8, 128 x 128 22 / 15, 512 x 32 19 / 17, 1024 x 8 19 / 13, 1024 x 16 18 / 16 (8 experts
+// a token: 18 / 20); past the line 3072 x 8 19 / 29 with 48 tokens a thread.
+constexpr int kSmallTokens = 16;  // tokens of one thread
 __host__ __device__ __forceinline__ int bucket_small_segs(int E) { return 1024 / E < 64 ? 1024 / E : 64; }
 
 template <int WDT>
@@ -329,15 +329,13 @@ __global__ __launch_bounds__(1024) void bucket_small_kernel(const void* __restri
   const int e = tid % E, seg = tid / E;
   const int t0 = seg * per;
   const int n = seg < nseg ? (T - t0 < per ? T - t0 : per) : 0;  // this thread's tokens (may be <= 0)
-  uint64_t nz = 0;
-  for (int j0 = 0; j0 < n; j0 += 16) {
-    float v[16];
+  float v[kSmallTokens];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = j0 + j < n ? load_as_f32<WDT>(w, (int64_t)(t0 + j0 + j) * E + e) : 0.f;
+  for (int j = 0; j < kSmallTokens; ++j) v[j] = j < n ? load_as_f32<WDT>(w, (int64_t)(t0 + j) * E + e) : 0.f;
+  int own = 0;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) nz |= (uint64_t)(v[j] != 0.f) << (j0 + j);
-  }
-  s_seg[tid] = __popcll(nz);
+  for (int j = 0; j < kSmallTokens; ++j) own += v[j] != 0.f;
+  s_seg[tid] = own;
   __syncthreads();
   int tot = 0;
   if (tid < E) {  // exclusive prefix over the expert's segments, in place
@@ -375,18 +373,19 @@ __global__ __launch_bounds__(1024) void bucket_small_kernel(const void* __restri
   }
   __syncthreads();
   int64_t pos = s_seg[tid];  // unclamped: only slots below capacity are stored
-  for (int j = 0; j < n; ++j) {
-    const int64_t at = (int64_t)(t0 + j) * E + e;
+#pragma unroll
+  for (int j = 0; j < kSmallTokens; ++j) {
+    if (j >= n) break;
     int32_t sl = -1;
-    if (nz >> j & 1) {
+    if (v[j] != 0.f) {
       if (pos < capacity) {
         token_idx[pos] = t0 + j;
-        slot_w[pos] = load_as_f32<WDT>(w, at);
+        slot_w[pos] = v[j];
         sl = (int32_t)pos;
       }
       ++pos;
     }
-    pair_slot[at] = sl;
+    pair_slot[(int64_t)(t0 + j) * E + e] = sl;
   }
   if (overflow)
     for (int64_t i = s_end + tid; i < capacity; i += 1024) {
@@ -901,7 +900,7 @@ extern "C" int usaf_hip_bucket_by_expert(const void* weights, int32_t weights_dt
   hipStream_t st = as_stream(stream);
   const int64_t n_chunks = (T + kChunk - 1) / kChunk;
   const int e = (int)E;
-  if (T > 0 && T * E <= kSmallPairs && T <= (int64_t)kSmallTokens * bucket_small_segs(e)) {
+  if (T > 0 && T <= (int64_t)kSmallTokens * bucket_small_segs(e)) {
     USAF_DISPATCH_DT(weights_dtype, WDT,
                      bucket_small_kernel<WDT><<<1, 1024, 0, st>>>(weights, (int)T, e, counts, offsets, capacity,
                                                                   token_idx, slot_w, pair_slot, overflow));
