@@ -60,3 +60,25 @@ def test_weight_grad_of_saved_tensors_in_another_layout(gpu_device):
         torch.cuda.synchronize()
         grads.append([q.grad for q in p])
     assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])
+
+
+@pytest.mark.parametrize("counts,R,C,out_dt", [
+    ([9000, 0, 5001], 72, 136, torch.bfloat16),  # 4 parts of each expert's slots
+    ([16411], 128, 64, torch.float32),  # 16 parts
+    ([4095], 64, 64, torch.float32),  # one slot short of 4 parts
+])
+def test_weight_grad_in_parts(gpu_device, counts, R, C, out_dt):
+    print(f"[gpu-case] weight grad in parts counts={counts} R={R} C={C} -> {out_dt}", flush=True)
+    gen = torch.Generator().manual_seed(R + C)
+    S, E = sum(counts), len(counts)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    # integers in [-4, 4]: sums of up to 16 * 16,411 are exact in fp32 in any order
+    dy = torch.randint(-4, 5, (S, R), generator=gen).to(torch.bfloat16)
+    x = torch.randint(-4, 5, (S, C), generator=gen).to(torch.bfloat16)
+    b = G.Buckets(None, offs.to(gpu_device), None, None, None, S)
+    out = G._dense_weight_grad(dy.to(gpu_device), x.to(gpu_device), None, b, out_dt)
+    torch.cuda.synchronize()
+    assert out.shape == (E, R, C) and out.dtype == out_dt and out.is_contiguous()
+    for e in range(E):
+        s = slice(int(offs[e]), int(offs[e + 1]))
+        assert torch.equal(out[e].cpu(), (dy[s].double().t() @ x[s].double()).to(out_dt)), e
