@@ -757,8 +757,8 @@ def probe_kernels(dev) -> None:
     torch.cuda.synchronize()
 
 
-KERNEL_SOURCES = ("usaf_amd/csrc/moe_gemm.hip", "usaf_amd/csrc/codec.hip", "usaf_amd/csrc/sparse.hip",
-                  "usaf_amd/csrc/common.h")
+KERNEL_SOURCES = ("usaf_amd/csrc/moe_gemm.hip", "usaf_amd/csrc/moe_gemm.h", "usaf_amd/csrc/codec.hip",
+                  "usaf_amd/csrc/sparse.hip", "usaf_amd/csrc/route.hip", "usaf_amd/csrc/common.h")
 
 
 def kernel_source_hash() -> str:
