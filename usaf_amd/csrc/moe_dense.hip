@@ -200,16 +200,6 @@ __global__ __launch_bounds__(DN_THREADS, 2) void moe_dense_kernel(const GemmArgs
             *reinterpret_cast<uint2*>(g.out2 + m * g.ldo2 + g.inter + n) = uint2{ub[0], ub[1]};
             *reinterpret_cast<uint2*>(g.out + m * g.ldo + n) = uint2{ab[0], ab[1]};
           }
-          if (g.out_t) {  // blocked act: feature rows of ld = round_up(se, 16) slots, zero past se
-            const int s0 = g.offsets[e], se = g.offsets[e + 1] - s0, ld = (se + 15) & ~15;
-            const int j = m_beg - s0 + 32 * i + l32;
-            if (j < ld) {
-              uint16_t* const dst = g.out_t + g.inter * (int64_t)g.blk_table[e] + n * ld + j;
-#pragma unroll
-              for (int c = 0; c < 4; ++c)
-                dst[c * (int64_t)ld] = live ? (uint16_t)(ab[c >> 1] >> (16 * (c & 1))) : (uint16_t)0;
-            }
-          }
         }
     } else if constexpr (WM == W_KN) {
       // the even columns are unit 0's rows, the odd ones unit 1's: 8 columns in a row
