@@ -176,12 +176,35 @@ def test_slot_cache_slots_beyond_4gib(gpu_device):
     slots = [cache.slot_of(name, e) for e in used]
     assert min(slots) >= 700 - len(used) and max(slots) == 699
     assert max(slots) * cache.gu_elems * 2 > 2 ** 32
-    check(f"out ({len(used)} experts in slots {min(slots)}..{max(slots)})", out,
-          M.experts_routed(x, w, deq[0].to(dt), deq[1].to(dt)), dt, say=_say)
+    ref = M.experts_routed(x, w, deq[0].to(dt), deq[1].to(dt))
+    check(f"out ({len(used)} experts in slots {min(slots)}..{max(slots)})", out, ref, dt, say=_say)
+    # three times the tokens, 108 slots per expert: past the short m-tile kernel's line of 96
+    out3 = cache.forward(name, x.repeat(3, 1).to(gpu_device), w.repeat(3, 1).to(gpu_device), k)
+    torch.cuda.synchronize()
+    check("out of the tokens three times", out3, ref.repeat(3, 1), dt, say=_say)
     for e in (used[0], used[-1]):
         s = cache.slot_of(name, e)
         assert torch.equal(cache.copy_of(s, "gate_up").cpu().view(torch.int16), deq[0][e].view(torch.int16))
         assert torch.equal(cache.copy_of(s, "down").cpu().view(torch.int16), deq[1][e].view(torch.int16))
+
+
+@pytest.mark.parametrize("T,k", [(154, 4), (153, 4)])
+def test_slot_cache_either_side_of_the_short_tile_line(gpu_device, T, k):
+    """T * (k + 1) slots for 8 experts: 96.25 each (persistent kernel) and 95.6 (short m-tiles)."""
+    E, H, I, dt = 8, 256, 128, torch.float16
+    _say(f"slot cache: E={E} H={H} I={I} T={T} k={k}, {T * (k + 1) / E:.1f} slots per expert")
+    g = torch.Generator().manual_seed(77)
+    qs = [G.Q4Tensor.quantize((torch.randn(shp, generator=g) * 0.02).half().to(gpu_device))
+          for shp in ((E, 2 * I, H), (E, H, I))]
+    deq = [torch.from_numpy(oracle.dequant(q.q.cpu().numpy(), q.s.cpu().numpy(), q.z.cpu().numpy(), q.numel(),
+                                           out_dtype="fp16").view(np.int16).copy()).view(dt).reshape(tuple(q.shape))
+           for q in qs]
+    cache = ExpertSlotCache({"l": G.ExpertWeights(*qs)}, gpu_device, max_bytes=E * cache_slot_bytes(H, I, dt), dtype=dt)
+    w, _, _ = M.route(torch.randn(T, E, generator=g), k, False, dt)
+    x = torch.randn(T, H, generator=g).to(dt)
+    out = cache.forward("l", x.to(gpu_device), w.to(gpu_device), k)
+    torch.cuda.synchronize()
+    check("out", out, M.experts_routed(x, w, *deq), dt, say=_say)
 
 
 def cache_slot_bytes(H, I, dt):

@@ -1,7 +1,8 @@
 """The grouped GEMMs on dense weights at short m-tiles (moe_dense.hip), in all
 three weight orders, where their tiles end: experts without slots, with 1, 31, 32,
 33, 95 to 97 and 127 to 129, one expert only, 255 experts, widths that leave waves
-without columns, one and odd counts of k-steps, weights behind a slot table.
+without columns, one and odd counts of k-steps, weights behind a slot table; and the
+persistent kernels (moe_gemm.hip) past the line of each order.
 
 Weights in [-8, 7] and activations in [-2, 2] are integers: every sum is exact in
 fp32 in any order, and outputs rounded once must equal the 64-bit product rounded
@@ -44,15 +45,35 @@ CASES = [  # E, H, I, slots of the experts in turn, dtype
 
 @pytest.mark.parametrize("E,H,I,slots,dt", CASES, ids=lambda v: None if isinstance(v, list) else str(v))
 def test_dense_slots(gpu_device, E, H, I, slots, dt):
+    counts = [slots[e % len(slots)] for e in range(E)]
+    assert 0 < sum(counts) <= 80 * E  # few enough for every order
+    _run(gpu_device, E, H, I, counts, dt)
+
+
+# slots per expert on either side of each order's line: rows 80, fragment 96, [K, N] 128
+@pytest.mark.parametrize("slots", [81, 96, 97, 128, 129, 321])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_dense_slots_lines(gpu_device, slots, dt):
+    _run(gpu_device, 3, 256, 384, [slots + 7, slots - 7, slots], dt)
+
+
+@pytest.mark.parametrize("H,I", [(64, 128), (192, 128), (128, 32), (256, 96), (128, 160)])
+def test_dense_slots_odd_k_steps(gpu_device, H, I):
+    """One and odd counts of 64-wide k-steps, and widths that leave waves without columns
+    (the GEMMs whose shapes take them)."""
+    _run(gpu_device, 3, H, I, [33, 0, 65], torch.bfloat16)
+
+
+def _run(gpu_device, E, H, I, counts, dt):
+    """Every GEMM whose shape allows H and I, against the 64-bit products."""
     dev = gpu_device
     gen = torch.Generator().manual_seed(E * 7 + H + I)
-    counts = [slots[e % len(slots)] for e in range(E)]
     S, T = sum(counts), 64
-    assert 0 < S <= 80 * E  # few enough for every order
     print(f"[gpu-case] dense slots E={E} H={H} I={I} S={S} {dt}", flush=True)
     ints = lambda lo, hi, *s: torch.randint(lo, hi + 1, s, generator=gen).to(dt)
     wg, wd = ints(-8, 7, E, 2 * I, H), ints(-8, 7, E, H, I)
     slot_of = torch.randperm(E + 3, generator=gen)[:E]
+    wide_h, wide_i = H % 128 == 0, I % 128 == 0  # contraction (gate_up; down) and down's activations
     offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
     tok = torch.randint(0, T, (S,), generator=gen).to(torch.int32)
     # x with about 32 non-zeros a row: gate * up stays below fp16's largest value
@@ -69,43 +90,54 @@ def test_dense_slots(gpu_device, E, H, I, slots, dt):
 
     d = {n: t.to(dev) for n, t in (("x", x), ("act", act_in), ("dcur", dcur), ("dgu", dgu_in), ("gu", gu_in),
                                    ("tok", tok), ("offs", offs), ("wg", wg), ("wd", wd),
-                                   ("ag", _arena(wg, I, slot_of, E + 3)), ("ad", _arena(wd, 0, slot_of, E + 3)),
                                    ("slot", slot_of.to(torch.int32)))}
+    if wide_h and wide_i:
+        d["ag"], d["ad"] = _arena(wg, I, slot_of, E + 3).to(dev), _arena(wd, 0, slot_of, E + 3).to(dev)
     empty = lambda *s: torch.full(s, float("nan"), dtype=dt, device=dev)
     code, st = N.dtype_code(dt), N.stream_ptr(dev)
     table = G.blocked_layout(d["offs"], S)
     blk = empty(int(N.load().usaf_hip_blocked_elems(S, E, I)))
     for order in ("rows", "fragment"):
+        if order == "fragment" and not (wide_h and wide_i):
+            continue
         gu, act, y = empty(S, 2 * I), empty(S, I), empty(S, H)
         if order == "rows":
-            N.call("usaf_hip_moe_gate_up_fwd", d["x"].data_ptr(), T, H, d["tok"].data_ptr(), d["offs"].data_ptr(), S, E,
-                   I, None, None, d["wg"].data_ptr(), code, gu.data_ptr(), act.data_ptr(), blk.data_ptr(),
-                   table.data_ptr(), None, 0, st)
-            N.call("usaf_hip_moe_down_fwd", d["act"].data_ptr(), I, d["offs"].data_ptr(), S, E, H, None, None,
-                   d["wd"].data_ptr(), code, y.data_ptr(), None, 0, st)
+            if wide_h:
+                N.call("usaf_hip_moe_gate_up_fwd", d["x"].data_ptr(), T, H, d["tok"].data_ptr(), d["offs"].data_ptr(),
+                       S, E, I, None, None, d["wg"].data_ptr(), code, gu.data_ptr(), act.data_ptr(), blk.data_ptr(),
+                       table.data_ptr(), None, 0, st)
+            if wide_i:
+                N.call("usaf_hip_moe_down_fwd", d["act"].data_ptr(), I, d["offs"].data_ptr(), S, E, H, None, None,
+                       d["wd"].data_ptr(), code, y.data_ptr(), None, 0, st)
         else:
             N.call("usaf_hip_moe_gate_up_fwd_slots", d["x"].data_ptr(), T, H, d["tok"].data_ptr(), d["offs"].data_ptr(),
                    S, E, I, d["ag"].data_ptr(), d["slot"].data_ptr(), E + 3, code, gu.data_ptr(), act.data_ptr(), st)
             N.call("usaf_hip_moe_down_fwd_slots", d["act"].data_ptr(), I, d["offs"].data_ptr(), S, E, H,
                    d["ad"].data_ptr(), d["slot"].data_ptr(), E + 3, code, y.data_ptr(), st)
         torch.cuda.synchronize()
-        assert torch.equal(gu.cpu(), exact(x[tok.long()], wg, True)), order
-        assert torch.equal(y.cpu(), exact(act_in, wd, True)), order
-        g, u = gu.cpu().double().split(I, 1)
-        assert close(act.cpu(), g * torch.sigmoid(g) * u, (g * u).abs()), order
-        if order == "rows":  # act's blocked copy, bit for bit
+        if wide_i:
+            assert torch.equal(y.cpu(), exact(act_in, wd, True)), order
+        if wide_h:
+            assert torch.equal(gu.cpu(), exact(x[tok.long()], wg, True)), order
+            g, u = gu.cpu().double().split(I, 1)
+            assert close(act.cpu(), g * torch.sigmoid(g) * u, (g * u).abs()), order
+        if wide_h and order == "rows":  # act's blocked copy (a transpose behind the GEMM), bit for bit
             want = G.slot_blocked(act, d["offs"], S, table=table).data
             n = int(((offs[1:] - offs[:-1] + 15) // 16 * 16).sum()) * I
             assert torch.equal(blk[:n].view(torch.int16), want[:n].view(torch.int16))
 
     dgu, dx = empty(S, 2 * I), empty(S, H)
-    N.call("usaf_hip_moe_down_bwd", d["dcur"].data_ptr(), H, d["gu"].data_ptr(), d["offs"].data_ptr(), S, E, I, None,
-           None, d["wd"].data_ptr(), code, dgu.data_ptr(), st)
-    N.call("usaf_hip_moe_gate_up_bwd", d["dgu"].data_ptr(), I, d["offs"].data_ptr(), S, E, H, None, None,
-           d["wg"].data_ptr(), code, dx.data_ptr(), st)
+    if wide_i:
+        N.call("usaf_hip_moe_down_bwd", d["dcur"].data_ptr(), H, d["gu"].data_ptr(), d["offs"].data_ptr(), S, E, I, None,
+               None, d["wd"].data_ptr(), code, dgu.data_ptr(), st)
+    if wide_h:
+        N.call("usaf_hip_moe_gate_up_bwd", d["dgu"].data_ptr(), I, d["offs"].data_ptr(), S, E, H, None, None,
+               d["wg"].data_ptr(), code, dx.data_ptr(), st)
     torch.cuda.synchronize()
-    assert torch.equal(dx.cpu(), exact(dgu_in, wg, False))
-    g, u = gu_in.double().split(I, 1)
-    da, sig = exact(dcur, wd, False).double(), torch.sigmoid(g)
-    assert close(dgu.cpu(), torch.cat([da * u * sig * (1 + g * (1 - sig)), da * g * sig], 1),
-                 torch.cat([(da * u).abs(), (da * g).abs()], 1))
+    if wide_h:
+        assert torch.equal(dx.cpu(), exact(dgu_in, wg, False))
+    if wide_i:
+        g, u = gu_in.double().split(I, 1)
+        da, sig = exact(dcur, wd, False).double(), torch.sigmoid(g)
+        assert close(dgu.cpu(), torch.cat([da * u * sig * (1 + g * (1 - sig)), da * g * sig], 1),
+                     torch.cat([(da * u).abs(), (da * g).abs()], 1))

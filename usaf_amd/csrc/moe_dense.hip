@@ -15,8 +15,9 @@
 // * NM = 4 (3 for [K, N], whose raw dwords and fragments would spill at 4: d(act) at
 //   64 slots 94 against 68 us).  A k-step (64 KB a CU) in flight does as
 //   well as three sets of registers at NM = 2 or 3 (153 against 155, 175 us).
-// Measured (OLMoE, 512 tokens, bf16, us, gate_up / down / d(act) / d(x); floor: the
-// weights at 6 TB/s, 89 / 45 / 45 / 89): 188 / 83 / 122 / 219 -> 153 / 67 / 68 / 131.
+// Measured (kernel trace of a training pass, OLMoE, 512 tokens, bf16, us, gate_up / down /
+// d(act) / d(x); floor: the weights at 6 TB/s, 89 / 45 / 45 / 89; before: the persistent
+// kernels): 188 / 82 / 124 / 227 -> 117 / 66 / 69 / 105.
 #include "moe_gemm.h"
 
 #include <type_traits>
@@ -270,13 +271,19 @@ int launch_dense_epi(const GemmArgs& g, int dt, int64_t S, hipStream_t st, const
 }  // namespace
 
 // The lines against the persistent kernels (moe_gemm.hip), in slots per expert on
-// average.  Measured, that kernel / this one, us:
-// * [N, K] rows, OLMoE gate_up + down: 269 / 205 at 8, 271 / 221 at 64, 288 / 316
-//   at 128 (experts past 128 slots take a second m-tile and read their weights again).
-// * Fragment order, passes of two Qwen3 layers: 772 / 682 at 64 slots with uniform
-//   popularity, 840 / 716 with Zipf; at 128 slots 849 / 883 and 936 / 933.
-// * [K, N], OLMoE d(x) + d(act): 337 / 179 at 8, 341 / 199 at 64, 366 / 307 at 128,
-//   402 / 475 at 256.
+// average.  Measured, those kernels / this one, us; a uniform routing, Zipf(1.1):
+// * [N, K] rows, gate_up + down with cold weights, 80 slots: OLMoE 244 / 185, 325 / 257,
+//   Qwen3 357 / 291, 422 / 378; warm, OLMoE at 128 slots, uniform: 288 / 316 (experts past
+//   128 slots take a second m-tile and read their weights again).
+// * Fragment order, passes of two Qwen3 layers: 772 / 682, 840 / 716 at 64 slots; at 128
+//   849 / 883, 956 / 877 and with another Zipf routing 936 / 933; at 256 1294 / 1321, 1277 / 1201.
+//   How the slots spread decides, which their average does not tell: the line stays
+//   where both win.
+// * [K, N], d(act) + d(x) with cold weights, 128 slots: OLMoE 367 / 304, 469 / 262, Qwen3
+//   511 / 447, 624 / 396; warm, OLMoE at 256 slots, uniform: 402 / 475.
+// With every token on the same eight experts a 128-slot m-tile reads their weights
+// more often than the persistent kernels' 256-slot ones: 640 OLMoE tokens, gate_up +
+// down 126 / 159 in rows, 103 / 123 in fragment order.
 bool dense_slots(const GemmArgs& g, int epi, bool kn, int64_t S, int64_t a_rows_total) {
   const int64_t lim = kn ? 128 : g.w_frag ? 96 : 80;
   const int64_t cols = epi == EPI_SWIGLU_FWD ? 32 : 64;
