@@ -1,5 +1,6 @@
-// What the grouped GEMM kernels share (moe_gemm.hip, moe_few.hip): operands,
-// epilogue codes, the 4-bit dequantization of a fragment and the MFMA.
+// What the grouped GEMM kernels share (moe_gemm.hip, moe_few.hip, moe_dense.hip,
+// wgrad.hip): operands, epilogue codes, the 4-bit dequantization of a fragment and
+// the MFMA.
 #pragma once
 
 #include "common.h"
