@@ -115,36 +115,52 @@ def test_few_slots(gpu_device, E, H, I, slots, dt, overlay):
     ("gate_up", 255, 160, 1536, [1, 0, 3]),  # split in two: the last block's second pair of waves has no rows
     ("gate_up", 8, 3008, 3072, [28, 33, 20]),  # four units a wave, split in four
     ("down", 8, 6016, 3072, [28, 33, 20]),
+    ("d_act", 128, 2048, 1536, [16, 5, 33]),  # four units a wave, transposed, through the SwiGLU backward
 ])
 def test_few_slots_one_gemm(gpu_device, gemm, E, cols, K, slots):
-    """cols columns from a contraction of K (gate_up: cols gate and cols up rows)."""
+    """cols columns from a contraction of K (gate_up: cols gate and cols up rows; d_act:
+    the gradients of gate and up from the transposed copy of a [K, cols] weight)."""
     dev, dt = gpu_device, torch.bfloat16
     gen = torch.Generator().manual_seed(E + cols + K)
     counts = [slots[e % len(slots)] for e in range(E)]
-    S, rows = sum(counts), 2 * cols if gemm == "gate_up" else cols
-    assert 0 < S <= 28 * E
+    S, rows, k = sum(counts), {"gate_up": 2 * cols, "down": cols, "d_act": K}[gemm], cols if gemm == "d_act" else K
+    assert 0 < S <= (20 if gemm == "d_act" else 28) * E
     print(f"[gpu-case] few slots {gemm} E={E} cols={cols} K={K} S={S}", flush=True)
-    q = torch.randint(-128, 128, (E, rows * K // 2), generator=gen, dtype=torch.int8)
-    one = torch.ones(E * rows * K // 128, dtype=torch.float16)
-    w = G.Q4Tensor(q.view(-1, 64).to(dev), one.to(dev), (-8 * one).to(dev), torch.Size((E, rows, K)), 128)
+    q = torch.randint(-128, 128, (E, rows * k // 2), generator=gen, dtype=torch.int8)
+    one = torch.ones(E * rows * k // 128, dtype=torch.float16)
+    w = G.Q4Tensor(q.view(-1, 64).to(dev), one.to(dev), (-8 * one).to(dev), torch.Size((E, rows, k)), 128)
     offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
     x = torch.randint(-2, 3, (S, K), generator=gen).to(dt)
-    d_x, d_offs, d_rows = x.to(dev), offs.to(dev), torch.arange(S, dtype=torch.int32, device=dev)
-    out = torch.full((S, rows), float("nan"), dtype=dt, device=dev)
+    gu = torch.randn(S, 2 * cols, generator=gen).to(dt)
+    d_x, d_offs, d_rows, d_gu = x.to(dev), offs.to(dev), torch.arange(S, dtype=torch.int32, device=dev), gu.to(dev)
+    out = torch.full((S, cols if gemm == "down" else 2 * cols), float("nan"), dtype=dt, device=dev)
     code, st = N.dtype_code(dt), N.stream_ptr(dev)
     if gemm == "gate_up":
         act = torch.empty(S, cols, dtype=dt, device=dev)
         N.call("usaf_hip_moe_gate_up_fwd", d_x.data_ptr(), S, K, d_rows.data_ptr(), d_offs.data_ptr(), S, E, cols,
                w.q.data_ptr(), w.scale_zero().data_ptr(), None, code, out.data_ptr(), act.data_ptr(), None, None,
                None, 0, st)
-    else:
+    elif gemm == "down":
         N.call("usaf_hip_moe_down_fwd", d_x.data_ptr(), K, d_offs.data_ptr(), S, E, cols, w.q.data_ptr(),
                w.scale_zero().data_ptr(), None, code, out.data_ptr(), None, 0, st)
+    else:
+        wt, szt = w.transposed()
+        N.call("usaf_hip_moe_down_bwd_t", d_x.data_ptr(), K, d_gu.data_ptr(), d_offs.data_ptr(), S, E, cols,
+               wt.data_ptr(), szt.data_ptr(), code, out.data_ptr(), None, 0, st)
     torch.cuda.synchronize()
     got = out.cpu()
     for e in range(E):
         a, b = int(offs[e]), int(offs[e + 1])
-        if a < b:
-            raw = q[e].view(torch.uint8)
-            vals = torch.stack([raw & 15, raw >> 4], 1).double().view(rows, K) - 8
+        if a == b:
+            continue
+        raw = q[e].view(torch.uint8)
+        vals = torch.stack([raw & 15, raw >> 4], 1).double().view(rows, k) - 8
+        if gemm != "d_act":
             assert torch.equal(got[a:b], (x[a:b].double() @ vals.t()).to(dt)), e
+            continue
+        da = (x[a:b].double() @ vals).to(dt).double()
+        g, u = gu[a:b].double().split(cols, 1)
+        sig = torch.sigmoid(g)
+        ref = torch.cat([da * u * sig * (1 + g * (1 - sig)), da * g * sig], 1)
+        tiny = float(torch.finfo(dt).tiny) * (1 + torch.cat([(da * u).abs(), (da * g).abs()], 1))
+        assert bool(((got[a:b].double() - ref).abs() <= EPS[dt] * ref.abs() + tiny).all()), e
